@@ -59,6 +59,7 @@ struct PlainArgs {
     int32_t listed;   // 1: the emission takes the listed tiles
     int32_t wpc;     // workgroups of 256 lines per chunk
     int32_t nx_tab;  // distinct x among a workgroup's lines, at most
+    int32_t zseg, zlen;  // z segments of a line (sample_density) and samples of each
     float step;
     const unsigned char* ztab;
     float* dens;
@@ -130,8 +131,16 @@ __device__ __forceinline__ void list_tiles(const PlainArgs& a, int32_t chunk, in
 // whatever the resolution (x-planes of their own leave 207 of 256 lanes idle at 49 samples per axis:
 // 73 -> 33 us for 48 chunks of 48^3 at 6 octaves); the x and y entries of its lines are in LDS.
 // BUILD: densities to the scratch layout, and sign words. !BUILD: densities to the caller's layout (z fastest),
-// through an LDS tile of 16 samples per line so that stores are 64-byte runs, and the sign summary.
+// through an LDS tile of 16 samples per line so that stores are 64-byte runs, and the sign summary. There a
+// workgroup may take a z segment of its lines (zseg > 1, uw_sample_density): a line's samples and tile
+// flushes are one chain, which is the launch's time while compute units stand idle.
 constexpr int kTileZ = 16, kTilePitch = kTileZ + 1;
+// Segments are cut while a launch has fewer than 2 workgroups per compute unit, to 8 samples at least:
+// each segment repeats the x and y entries of its lines and builds every octave's lattice faces at its
+// first sample (6 octaves: 8 chunks of 64^3 41.9 -> 24.6 us, 64 of 32^3 32.5 -> 25.2, 64 of 8^3 19.6 ->
+// 15.8; cut up to 4 per unit, 24 of 64^3 took 42.9 where 2 take 33.1, and 256 of 24^3 37.2 where uncut
+// lines take 30.6).
+constexpr int kSegPerCu = 2, kSegSamples = 8;
 
 template <int OCT, bool BUILD>
 __global__ void __launch_bounds__(kThreads) k_lines(PlainArgs a) {
@@ -147,7 +156,12 @@ __global__ void __launch_bounds__(kThreads) k_lines(PlainArgs a) {
     __shared__ uint32_t s_bits;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int nthr = int(blockDim.x);  // 256, or the waves that one chunk's lines fill
-    const int32_t chunk = int32_t(blockIdx.x) / a.wpc, t0 = (int32_t(blockIdx.x) - chunk * a.wpc) * nthr;
+    int32_t item = int32_t(blockIdx.x), seg = 0;
+    if (!BUILD) {
+        item = int32_t(blockIdx.x) / a.zseg;
+        seg = int32_t(blockIdx.x) - item * a.zseg;
+    }
+    const int32_t chunk = item / a.wpc, t0 = (item - chunk * a.wpc) * nthr;
     const int32_t cx = a.coords[3 * chunk], cy = a.coords[3 * chunk + 1];
     if (tid == 0) s_bits = 0u;
     if (tid < UW_MAX_OCTAVES) s_freq[tid] = a.f.octave_freq[tid];
@@ -208,27 +222,33 @@ __global__ void __launch_bounds__(kThreads) k_lines(PlainArgs a) {
             }
             bits = (vmin <= iso ? UW_BELOW_NOT_ABOVE : 0u) | (any ? UW_BELOW_LT : 0u) | (~all ? UW_BELOW_GE : 0u);
         } else {
-            float* dst = a.dens + (uint64_t(chunk) * uint64_t(lines) + uint64_t(t0 + 64 * wave)) * uint64_t(L);
+            const int32_t z0 = seg * a.zlen, count = min(L - z0, a.zlen);
+            float* dst = a.dens + (uint64_t(chunk) * uint64_t(lines) + uint64_t(t0 + 64 * wave)) * uint64_t(L) + z0;
             float* tile = TILE + wave * 64 * kTilePitch;
             const int32_t left = lines - (t0 + 64 * wave);  // lines of the wave
-            // samples [z0, z0 + nz) of the wave's lines, from its tile (LDS operations of a wave stay in order)
-            auto flush = [&](int32_t z0, int32_t nz) {
+            // samples [z, z + nz) of the segment from the wave's tile, 64 at a time over its lines (LDS
+            // operations of a wave stay in order)
+            auto flush = [&](int32_t z, int32_t nz, const uw_divider& dn) {
                 __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
                 __builtin_amdgcn_wave_barrier();
-                const int32_t z = lane & (kTileZ - 1);
 #pragma unroll 4
-                for (int32_t q = lane / kTileZ; q < 64; q += 64 / kTileZ)
-                    if (q < left && z < nz) dst[q * L + z0 + z] = tile[q * kTilePitch + z];
+                for (int32_t i = 0; i < nz; ++i) {
+                    const uint32_t e = uint32_t(64 * i + lane);
+                    const int32_t q = int32_t(uw_div(e, dn)), k = int32_t(e) - q * nz;
+                    if (q < left) dst[q * L + z + k] = tile[q * kTilePitch + k];
+                }
                 __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
                 __builtin_amdgcn_wave_barrier();
             };
-            uw_noise_zline<OCT, false>(
-                a.f, [=](int k) { return ax[k]; }, [=](int k) { return ay[k]; }, P, GH, Zt.rec, rw, L, vmin,
+            const uw_divider dfull = uw_make_divider(kTileZ);
+            uw_noise_zline<OCT, true>(
+                a.f, [=](int k) { return ax[k]; }, [=](int k) { return ay[k]; }, P, GH, Zt.rec + z0 * rw, rw, count, vmin,
                 vmax, [&](int32_t iz, float rho) {
                     tile[lane * kTilePitch + (iz & (kTileZ - 1))] = rho;
-                    if ((iz & (kTileZ - 1)) == kTileZ - 1) flush(iz - (kTileZ - 1), kTileZ);
+                    if ((iz & (kTileZ - 1)) == kTileZ - 1) flush(iz - (kTileZ - 1), kTileZ, dfull);
                 });
-            if (L & (kTileZ - 1)) flush(L & ~(kTileZ - 1), L & (kTileZ - 1));
+            const int32_t rest = count & (kTileZ - 1);
+            if (rest) flush(count - rest, rest, uw_make_divider(uint32_t(rest)));
             bits = uint32_t(uw_below_bits(vmin, vmax, iso));
         }
     }
@@ -560,6 +580,8 @@ int plain_args(uw_ctx* ctx, const int32_t* coords, int32_t nchunks, int32_t n, i
     a->wpc = (a->L * a->L + kThreads - 1) / kThreads;
     a->nx_tab = (kThreads - 1) / a->L + 2;
     if (a->nx_tab > a->L) a->nx_tab = a->L;
+    a->zseg = 1;
+    a->zlen = a->L;
     a->step = float(a->f.extent) / float(n);
     a->ztab = base + lay->ztab;
     a->ngroups = lay->ngroups;
@@ -578,7 +600,7 @@ int plain_args(uw_ctx* ctx, const int32_t* coords, int32_t nchunks, int32_t n, i
 int launch_lines(uw_ctx* ctx, const PlainArgs& a, const PlainLayout& lay, LinesKernel k, bool build, hipStream_t st) {
     const int32_t O = a.f.octaves;
     const uint64_t zblocks = (uint64_t(a.nchunks) * uint64_t(a.L + 1) + kThreads - 1) / kThreads;
-    const uint64_t blocks = uint64_t(a.nchunks) * uint64_t(a.wpc);
+    const uint64_t blocks = uint64_t(a.nchunks) * uint64_t(a.wpc) * uint64_t(a.zseg);
     if (zblocks > 0x7FFFFFFFull || blocks > 0x7FFFFFFFull) return uw_fail(ctx, UW_ERR_INVALID_ARG, "too many chunks for one launch");
     const size_t lds = lines_lds_bytes(O, a.L, a.nx_tab, build);
     UW_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
@@ -612,6 +634,13 @@ int uw_sample_density(uw_ctx* ctx, const int32_t* coords, int32_t nchunks, int32
     if (int rc = plain_args(ctx, coords, nchunks, n, 0, &a, &lay)) return rc;
     a.dens = dens;
     if (below) a.below = below;
+    const int64_t want = int64_t(kSegPerCu) * ctx->num_cus, have = int64_t(nchunks) * a.wpc;
+    if (have < want) {
+        const int64_t most = (a.L + kSegSamples - 1) / kSegSamples, segs = (want + have - 1) / have;
+        a.zseg = int32_t(segs < most ? segs : most);
+        a.zlen = (a.L + a.zseg - 1) / a.zseg;
+        a.zseg = (a.L + a.zlen - 1) / a.zlen;
+    }
     return launch_lines(ctx, a, lay, pick_lines<false>(a.f.octaves), false, st);
 }
 
