@@ -662,12 +662,18 @@ int uw_build_chunks_plain(uw_ctx* ctx, const int32_t* coords, int32_t nchunks, i
         return UW_OK;
     }
     // slabs as deep as a tile takes (each repeats a halo plane and the fixed chain of passes), and
-    // shallower while a launch has fewer than 16 tiles per compute unit: most tiles hold no surface,
-    // and then the fullest tile's time is the launch's (48 chunks of 48^3: 32.1 us at 64 tiles per
-    // chunk, 24.8 at 192; now 24.2 at 64, 20.6 at 128 and 17.5 at 192)
+    // shallower while a launch has too few tiles to even out: most tiles hold no surface, and then the
+    // fullest tile's time is the launch's (48 chunks of 48^3: 32.1 us at 64 tiles per chunk, 24.8 at 192;
+    // now 24.2 at 64, 20.6 at 128 and 17.5 at 192). 16 per compute unit for tiles of many rows and for
+    // chunks of more than one row segment, a part of whose tiles is next to empty (64 chunks of 33^3: the
+    // launch 53.6 us at 8 per unit, 49.7 at 16); 8 for tiles of up to 150 rows, whose fixed chain outweighs
+    // their own share (1024 chunks: 4^3 36.7 us at 16 per unit, 30.9 at 8, 8^3 43.6 and 36.1, 12^3 50.3
+    // and 43.9; 512 of 12^3 44.6 and 35.4)
     int32_t planes = uw_tile_planes(n);
     uw_tiling tiling = uw_tiling_for(n, planes);
-    while (planes > 1 && int64_t(nchunks) * tiling.tiles() < 16 * int64_t(ctx->num_cus)) {
+    while (planes > 1) {
+        const int64_t want = (tiling.T > 1 || tiling.max_rows > 150 ? 16 : 8) * int64_t(ctx->num_cus);
+        if (int64_t(nchunks) * tiling.tiles() >= want) break;
         planes = (planes + 1) / 2;
         tiling = uw_tiling_for(n, planes);
     }
