@@ -7,7 +7,8 @@
 //                  (chunk.rs:141-164): one wave per chunk, or one workgroup above 32 cells per axis
 //   k_emit         one workgroup per (chunk, tile): the chunk's place in the output (sum of the sizes
 //                  before it), then vertices, indices and collision records (chunk.rs:164-250); the
-//                  first workgroups write the chunks' records and the totals
+//                  first workgroups write the chunks' records and the totals, and the cube cases of
+//                  every cell where the caller asks for them
 //
 // HBM layout (scratch, per chunk c of resolution n, L = n + 1):
 //   dens   [c][L^3] f32     sample (x, y, z) at z L^2 + x L + y: a wave's store is one row of lines
@@ -77,6 +78,8 @@ struct PlainArgs {
     uint32_t* inds;
     uw_emit_opts eo;
     uw_tiling tiling;
+    uint8_t* cases;     // cube cases of every cell (null: not asked for)
+    int32_t ncase;      // workgroups of the emission that write them
 };
 
 // A chunk's record (its offsets are the emission's) and its sizes, by one thread.
@@ -390,9 +393,37 @@ __device__ __forceinline__ void group_records(const PlainArgs& a, int32_t grp) {
     }
 }
 
-// Emission. Workgroups [0, groups) write the records. The others take tiles: LISTED, as many
-// workgroups as stay resident take the listed tiles (those with triangles), most triangles first, in
-// rounds of alternating direction so that the workgroups' sums stay even (a queue's claims, one atomic
+// Cube cases of every cell (chunk.rs:155-162), a row segment per thread and step, by workgroup b of
+// a.ncase: a launch of its own, one cell per thread, cost 1024 chunks of 8^3 cells 4.0 us and could not
+// hold 2^32 cells. Rows of a multiple of four cells are written in words.
+__device__ __forceinline__ void write_cases(const PlainArgs& a, uint32_t b) {
+    const uint32_t per = uint32_t(a.n) * uint32_t(a.n) * uint32_t(a.T);
+    const uint64_t rows = uint64_t(per) * uint64_t(a.nchunks);
+    const bool aligned = ((reinterpret_cast<uint64_t>(a.cases) | uint64_t(a.n)) & 3u) == 0u;
+    for (uint64_t r = uint64_t(b) * kThreads + threadIdx.x; r < rows; r += uint64_t(a.ncase) * kThreads) {
+        const uint64_t chunk = r / per;
+        const uint32_t s = uint32_t(r - chunk * per), q = s / uint32_t(a.T), x = q / uint32_t(a.n);
+        const int32_t tz = int32_t(s - q * uint32_t(a.T)), y = int32_t(q - x * uint32_t(a.n));
+        uw_row_bits w;
+        w.load(a.words + chunk * uint64_t(a.L * a.L) * a.WL, int32_t(x), y, tz, a.n, a.L, a.WL);
+        uint8_t* out = a.cases + (chunk * uint64_t(a.n * a.n) + q) * uint64_t(a.n) + 32 * tz;
+        const uint32_t nz = uint32_t(min(32, a.n - 32 * tz));
+        if (aligned) {
+            for (uint32_t z = 0; z < nz; z += 4) {
+                uint32_t v = 0;
+#pragma unroll
+                for (uint32_t i = 0; i < 4; ++i) v |= uw_case_of_index(w.index(z + i)) << (8 * i);
+                *reinterpret_cast<uint32_t*>(out + z) = v;
+            }
+        } else {
+            for (uint32_t z = 0; z < nz; ++z) out[z] = uint8_t(uw_case_of_index(w.index(z)));
+        }
+    }
+}
+
+// Emission. Workgroups [0, groups) write the records, the next ncase the cube cases. The others take
+// tiles: LISTED, as many workgroups as stay resident take the listed tiles (those with triangles), most
+// triangles first, in rounds of alternating direction so that the workgroups' sums stay even (a queue's claims, one atomic
 // per tile on one address, cost more than the balance they bring: 40 -> 54 us for 4096 chunks of
 // 12^3); else, for launches whose tiles all fit the device at once, workgroup b takes tile b, which
 // saves the look-ups. A chunk's first vertex and index are summed from the sizes before it (the groups
@@ -405,8 +436,13 @@ __global__ void __launch_bounds__(kThreads, EXTRA ? 5 : 6) k_emit(PlainArgs a) {
         group_records(a, int32_t(blockIdx.x));
         return;
     }
+    if (int32_t(blockIdx.x) < a.ngroups + a.ncase) {
+        write_cases(a, blockIdx.x - uint32_t(a.ngroups));
+        return;
+    }
     const int tid = threadIdx.x;
-    const uint32_t tiles = uint32_t(a.tiling.tiles()), G = gridDim.x - uint32_t(a.ngroups), b = blockIdx.x - uint32_t(a.ngroups);
+    const uint32_t before = uint32_t(a.ngroups) + uint32_t(a.ncase);
+    const uint32_t tiles = uint32_t(a.tiling.tiles()), G = gridDim.x - before, b = blockIdx.x - before;
     uint32_t ends[kTileClasses], items = 0;  // listed tiles of the classes up to each
     if (LISTED) {
 #pragma unroll
@@ -483,19 +519,6 @@ using EmitKernel = void (*)(PlainArgs);
 
 // Page-locked room for a host build's record and arrays (a full 12^3 chunk has 0.3 MB)
 constexpr uint64_t kChunkPinned = uint64_t(2) << 20;
-
-// Cube cases of every cell (chunk.rs:155-162), one thread per cell, for callers that ask for them.
-__global__ void __launch_bounds__(kThreads) k_cases(PlainArgs a, uint8_t* __restrict__ cases) {
-    const uint64_t g = uint64_t(blockIdx.x) * kThreads + threadIdx.x;
-    const uint64_t C = uint64_t(a.n) * a.n * a.n;
-    if (g >= C * uint64_t(a.nchunks)) return;
-    const uint64_t chunk = g / C;
-    const uint32_t cell = uint32_t(g - chunk * C), z = cell % uint32_t(a.n), q = cell / uint32_t(a.n);
-    const uint32_t y = q % uint32_t(a.n), x = q / uint32_t(a.n);
-    uw_row_bits b;
-    b.load(a.words + chunk * uint64_t(a.L * a.L) * a.WL, int32_t(x), int32_t(y), int32_t(z >> 5), a.n, a.L, a.WL);
-    cases[g] = uint8_t(uw_case_of_index(b.index(z & 31u)));
-}
 
 // LDS bytes of k_lines.
 size_t lines_lds_bytes(int32_t O, int32_t L, int32_t nx_tab, bool build) {
@@ -690,9 +713,6 @@ int uw_build_chunks_plain(uw_ctx* ctx, const int32_t* coords, int32_t nchunks, i
     a.verts = out->verts;
     a.inds = out->inds;
     a.eo = uw_make_emit_opts(out);
-    const uint64_t cblocks = (uint64_t(nchunks) * uint64_t(n) * n * n + kThreads - 1) / kThreads;
-    if (cases && cblocks > 0x7FFFFFFFull)
-        return uw_fail(ctx, UW_ERR_INVALID_ARG, "too many chunks for one launch");
     const size_t elds = uw_emit_lds_bytes(tiling.max_rows, tiling.cells);
     const bool extra = uw_emit_extra(a.eo);
     const EmitKernel listed = extra ? k_emit<true, true> : k_emit<true, false>, all = extra ? k_emit<false, true> : k_emit<false, false>;
@@ -716,12 +736,17 @@ int uw_build_chunks_plain(uw_ctx* ctx, const int32_t* coords, int32_t nchunks, i
         hipLaunchKernelGGL(k_rows_block, dim3(uint32_t(nchunks)), dim3(kRowsBlock), lds, st, a);
     }
     if (int rc = uw_prof_end(ctx, st)) return rc;
-    if (cases) hipLaunchKernelGGL(k_cases, dim3(uint32_t(cblocks)), dim3(kThreads), 0, st, a, cases);
+    if (cases) {  // as many workgroups as the cases fill, at most 4 per compute unit
+        const uint64_t blocks = (uint64_t(nchunks) * uint64_t(n) * n * a.T + kThreads - 1) / kThreads, most = 4 * uint64_t(ctx->num_cus);
+        a.cases = cases;
+        a.ncase = int32_t(blocks < most ? blocks : most);
+    }
+    const uint32_t first = uint32_t(lay.ngroups) + uint32_t(a.ncase);  // workgroups before the tiles'
     if (int rc = uw_prof_start(ctx, st, UW_STAGE_PLAIN_EMIT)) return rc;
     if (!a.listed)
-        hipLaunchKernelGGL(all, dim3(uint32_t(lay.ngroups) + uint32_t(items)), dim3(kThreads), elds, st, a);
+        hipLaunchKernelGGL(all, dim3(first + uint32_t(items)), dim3(kThreads), elds, st, a);
     else
-        hipLaunchKernelGGL(listed, dim3(uint32_t(lay.ngroups) + uint32_t(resident)), dim3(kThreads), elds, st, a);
+        hipLaunchKernelGGL(listed, dim3(first + uint32_t(resident)), dim3(kThreads), elds, st, a);
     if (int rc = uw_prof_end(ctx, st)) return rc;
     UW_HIP(ctx, hipGetLastError());
     return UW_OK;
