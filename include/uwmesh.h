@@ -237,8 +237,10 @@ int uw_tris_around(const uint32_t* tri_cells, uint32_t ntris, int32_t n, float p
  * axis (slab[n] = n builds the chunk in one slab with one density evaluation; smaller slabs bound
  * LDS use and evaluate the densities twice); bulk_min: chunks of at least bulk_min cells per axis
  * (up to max_res) leave the persistent queue for the bulk path, whose launches spread each chunk's
- * lines, rows and tiles over the device (1, the default: every chunk, with no persistent launch; 0 or a
- * value above max_res: no bulk path). */
+ * lines, rows and tiles over the device (1, the default: every chunk, with no persistent launch, except
+ * that at 3, 4, 6 or 8 octaves a launch of plain vertices and u32 indices whose chunks are each built in
+ * one pass and have a workgroup of their own stays on the persistent kernel, where it takes two launches
+ * instead of four; 0 or a value above max_res: no bulk path). */
 typedef struct uw_batch_tuning {
     int32_t block;
     int32_t grid;

@@ -41,7 +41,8 @@ constexpr int kDensBudget = 20 * 1024;  // default LDS bytes for the density sla
 // over the device, the persistent kernel holds a whole chunk in one workgroup): 41 us of kernels against
 // 75 for a world update, 98 against 196 for 1000 chunks of 3 .. 32 cells, 517 against 577 for 8192 of
 // 8 .. 32, a launch of 4096 of 12^3 at 3 octaves 91 against 121. The persistent kernel is left with
-// launches whose bulk scratch would pass its limit, and with a larger bulk_min set by the caller.
+// launches of few small chunks (few_small), those whose bulk scratch would pass its limit, and a larger
+// bulk_min set by the caller.
 constexpr int kDefaultBulkMin = 1;
 
 struct BatchArgs {
@@ -968,6 +969,7 @@ BatchedKernel pick_octaves(int octaves) {
         default: return k_batched<BLOCK, 0>;
     }
 }
+bool exact_octaves(int octaves) { return octaves == 3 || octaves == 4 || octaves == 6 || octaves == 8; }
 
 BatchedKernel pick_kernel(int block, int octaves) {
     switch (block) {
@@ -1051,12 +1053,44 @@ struct BatchLaunch {
 // Every chunk takes the bulk path.
 bool bulk_all(const uw_ctx* ctx, const uw_bulk_shape& s) { return s.on && ctx->batch_tuning.bulk_min == 1; }
 
+size_t persistent_lds(const uw_batch_tuning& t, int octaves, int32_t list_cap, int32_t ring, bool one_pass) {
+    return lds_fixed_bytes(size_t(list_cap), size_t(ring), one_pass ? 0 : 1) + lds_table_bytes(octaves, t.max_res + 1) +
+           dens_bytes_for(t);
+}
+
+// Launches that keep to the persistent kernel whatever bulk_min says: every chunk is built in one pass by
+// a workgroup of its own at the launch's start, at an octave count that has a kernel of its own. Their
+// time is the latency of the launches one after another, two where the bulk path has four (and host time
+// 5.9 us a call where that has 11 to 20). 4 octaves, 24 / 128 / 512 / 1000 chunks, kernels and gaps: 8^3
+// 24.4 / 24.8 / 26.0 / 30.0 us against 25.8 / 26.4 / 28.4 / 32.4 on the bulk path, 6^3 21.4 / 21.7 /
+// 23.9 / 28.8 against 25.4 / 25.7 / 27.4 / 29.4, 12^3 32.0 / 32.4 / 33.1 / 38.2 against 31.4 / 32.5 /
+// 34.5 / 37.3. Past that (1100 chunks of 8^3 at 3 octaves 31.7 against 32.9, 1400 39.3 and 33.8), with
+// colours, u16 indices or collision records (24 of 12^3 62 against 42) and on the kernel for any octave
+// count (128 of 8^3 28 against 23) the bulk path is the faster one.
+int few_small(uw_ctx* ctx, int32_t nchunks, bool extra, bool* yes) {
+    const uw_batch_tuning& t = ctx->batch_tuning;
+    const int32_t octaves = ctx->params.octaves, list_cap = list_cap_for(t);
+    *yes = false;
+    if (extra || !exact_octaves(octaves) || !one_pass_only(t, list_cap)) return UW_OK;
+    int per_cu = 0;
+    if (int rc = uw_resident(ctx, reinterpret_cast<const void*>(pick_kernel(t.block, octaves)), t.block,
+                             persistent_lds(t, octaves, list_cap, list_cap, true), &per_cu))
+        return rc;
+    *yes = per_cu > 0 && nchunks <= (t.grid > 0 ? t.grid : per_cu * ctx->num_cus);
+    return UW_OK;
+}
+
 // Launch shape of a batched launch (kernel, LDS, grid, ring, scratch sizes); allocates nothing.
-// allow_bulk = false keeps every chunk on the persistent kernel.
-int shape_batched(uw_ctx* ctx, int32_t nchunks, BatchLaunch* bl, bool allow_bulk = true) {
+// allow_bulk = false keeps every chunk on the persistent kernel. extra: uw_emit_extra of the output.
+int shape_batched(uw_ctx* ctx, int32_t nchunks, bool extra, BatchLaunch* bl, bool allow_bulk = true) {
     const int32_t octaves = ctx->params.octaves;
     bl->ztab_bytes = size_t(nchunks) * uw_ztab_bytes(octaves, ctx->batch_tuning.max_res + 1);
     memset(&bl->bulk, 0, sizeof(bl->bulk));
+    if (allow_bulk && ctx->batch_tuning.bulk_min == 1) {
+        bool few = false;
+        if (int rc = few_small(ctx, nchunks, extra, &few)) return rc;
+        allow_bulk = !few;
+    }
     if (allow_bulk)
         if (int rc = uw_bulk_shape_for(ctx, ctx->batch_tuning, nchunks, &bl->bulk)) return rc;
     bl->pt = ctx->batch_tuning;
@@ -1073,8 +1107,7 @@ int shape_batched(uw_ctx* ctx, int32_t nchunks, BatchLaunch* bl, bool allow_bulk
     bl->k = pick_kernel(tune.block, octaves);
     const int32_t list_cap = list_cap_for(tune);
     const bool one_pass = one_pass_only(tune, list_cap);
-    const size_t rest = lds_table_bytes(octaves, tune.max_res + 1) + dens_bytes_for(tune);
-    auto lds_for = [&](int32_t ring) { return lds_fixed_bytes(size_t(list_cap), size_t(ring), one_pass ? 0 : 1) + rest; };
+    auto lds_for = [&](int32_t ring) { return persistent_lds(tune, octaves, list_cap, ring, one_pass); };
     auto fits_per_cu = [&](size_t lds, int* per_cu) -> int {
         *per_cu = 0;
         if (int rc = uw_resident(ctx, reinterpret_cast<const void*>(bl->k), tune.block, lds, per_cu)) return rc;
@@ -1110,8 +1143,8 @@ int shape_batched(uw_ctx* ctx, int32_t nchunks, BatchLaunch* bl, bool allow_bulk
 }
 
 // shape_batched plus the context-owned scratch of the eager path (grown as needed).
-int prepare_batched(uw_ctx* ctx, int32_t nchunks, BatchLaunch* bl) {
-    if (int rc = shape_batched(ctx, nchunks, bl)) return rc;
+int prepare_batched(uw_ctx* ctx, int32_t nchunks, const uw_mesh_out* out, BatchLaunch* bl) {
+    if (int rc = shape_batched(ctx, nchunks, uw_emit_extra(uw_make_emit_opts(out)), bl)) return rc;
     if (size_t(nchunks) > ctx->batch_order_cap) {
         (void)hipFree(ctx->d_batch_order);
         ctx->d_batch_order = nullptr;
@@ -1254,7 +1287,7 @@ int uw_build_chunks_batched(uw_ctx* ctx, const int32_t* coords, const int32_t* r
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (int rc = uw_refuse_capture(ctx, st)) return rc;
     BatchLaunch bl;
-    if (int rc = prepare_batched(ctx, nchunks > 0 ? nchunks : 1, &bl)) return rc;
+    if (int rc = prepare_batched(ctx, nchunks > 0 ? nchunks : 1, out, &bl)) return rc;
     if (nchunks == 0) {
         hipLaunchKernelGGL(k_reset, dim3(1), dim3(64), 0, st, ctx->d_batch_head, out->totals);
         UW_HIP(ctx, hipGetLastError());
@@ -1273,7 +1306,7 @@ int uw_build_chunks_batched_tape(uw_ctx* ctx, const int32_t* coords, const int32
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (int rc = uw_refuse_capture(ctx, st)) return rc;
     BatchLaunch bl;
-    if (int rc = prepare_batched(ctx, nchunks > 0 ? nchunks : 1, &bl)) return rc;
+    if (int rc = prepare_batched(ctx, nchunks > 0 ? nchunks : 1, out, &bl)) return rc;
     if (nchunks == 0) {
         hipLaunchKernelGGL(k_reset, dim3(1), dim3(64), 0, st, ctx->d_batch_head, out->totals);
         UW_HIP(ctx, hipGetLastError());
@@ -1303,7 +1336,7 @@ int uw_batched_graph_create(uw_ctx* ctx, const int32_t* coords, const int32_t* r
     if (nchunks < 1 || !args_ok(nchunks, coords, res, out)) return uw_fail(ctx, UW_ERR_INVALID_ARG, "bad arguments");
     UW_HIP(ctx, hipSetDevice(ctx->device));
     BatchLaunch bl;
-    if (int rc = prepare_batched(ctx, nchunks, &bl)) return rc;
+    if (int rc = prepare_batched(ctx, nchunks, out, &bl)) return rc;
     // the graph owns its queue state, task records and z tables (the context's may be reallocated):
     // queue state at byte 0, task records (with the ordering keys and histograms) after it, z tables
     // after them, then the x-slab density scratch and the bulk path's scratch
@@ -1407,7 +1440,7 @@ int uw_build_chunks_batched_noalloc(uw_ctx* ctx, const int32_t* coords, const in
     if (!base) return uw_fail(ctx, UW_ERR_INVALID_ARG, "no-allocation scratch not set up on this device");
     hipStream_t st = static_cast<hipStream_t>(stream);
     BatchLaunch bl;
-    if (int rc = shape_batched(ctx, nchunks > 0 ? nchunks : 1, &bl, false)) return rc;
+    if (int rc = shape_batched(ctx, nchunks > 0 ? nchunks : 1, false, &bl, false)) return rc;
     const size_t need = noalloc_bytes(bl, nchunks > 0 ? nchunks : 1);
     if (need > kNoAllocBytes)
         return uw_fail(ctx, UW_ERR_INVALID_ARG,
