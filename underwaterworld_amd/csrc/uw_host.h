@@ -50,6 +50,6 @@ int uw_set_coord_launch(uw_ctx* ctx, int32_t* d_coord, int32_t x, int32_t y, int
 // kBlocksCount blocks, the rest is freed at once. A block may still be read by work queued before it was
 // given back: a taker synchronises the device after the take and before it writes.
 constexpr size_t kBlocksMax = size_t(256) << 20, kBlocksCount = 64;
-void* uw_block_take(uw_ctx* ctx, size_t bytes, size_t* got);
+int uw_block_take(uw_ctx* ctx, size_t bytes, void** out, size_t* got);
 void uw_block_give(uw_ctx* ctx, void* p, size_t bytes);
 void uw_host_release(uw_ctx* ctx);

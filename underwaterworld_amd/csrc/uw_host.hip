@@ -96,7 +96,7 @@ int uw_set_coord_launch(uw_ctx* ctx, int32_t* d_coord, int32_t x, int32_t y, int
     return UW_OK;
 }
 
-void* uw_block_take(uw_ctx* ctx, size_t bytes, size_t* got) {
+int uw_block_take(uw_ctx* ctx, size_t bytes, void** out, size_t* got) {
     {
         std::lock_guard<std::mutex> lock(ctx->host_lock);
         size_t best = ctx->blocks.size();
@@ -109,12 +109,13 @@ void* uw_block_take(uw_ctx* ctx, size_t bytes, size_t* got) {
             ctx->blocks.erase(ctx->blocks.begin() + std::ptrdiff_t(best));
             ctx->blocks_bytes -= b.bytes;
             *got = b.bytes;
-            return b.p;
+            *out = b.p;
+            return UW_OK;
         }
     }
-    void* p = nullptr;
+    *out = nullptr;
     *got = bytes;
-    if (hipMalloc(&p, bytes) == hipSuccess) return p;
+    if (hipMalloc(out, bytes) == hipSuccess) return UW_OK;
     (void)hipGetLastError();
     {  // the kept blocks may be what is missing
         std::lock_guard<std::mutex> lock(ctx->host_lock);
@@ -122,7 +123,12 @@ void* uw_block_take(uw_ctx* ctx, size_t bytes, size_t* got) {
         ctx->blocks.clear();
         ctx->blocks_bytes = 0;
     }
-    return hipMalloc(&p, bytes) == hipSuccess ? p : nullptr;
+    const hipError_t e = hipMalloc(out, bytes);
+    if (e == hipSuccess) return UW_OK;
+    (void)hipGetLastError();  // reported here, not by the next launch
+    *out = nullptr;
+    *got = 0;
+    return uw_hip_fail(ctx, e, "hipMalloc");
 }
 
 void uw_block_give(uw_ctx* ctx, void* p, size_t bytes) {

@@ -243,8 +243,7 @@ int ensure_staging(uw_world* w, int32_t k) {
     const uw_mesh_sections s = uw_sections(vcap, icap, format_of(w->cfg));
     const uint64_t in = (n * 4 * sizeof(int32_t) + 255) & ~uint64_t(255);
     const uint64_t rec = (sizeof(uw_totals) + n * sizeof(uw_chunk_info) + 255) & ~uint64_t(255);
-    w->stage = uw_block_take(w->ctx, in + rec + s.total, &w->stage_bytes);
-    if (!w->stage) return uw_fail(w->ctx, UW_ERR_HIP, "no device memory for a world batch");
+    if (int rc = uw_block_take(w->ctx, in + rec + s.total, &w->stage, &w->stage_bytes)) return rc;
     unsigned char* base = static_cast<unsigned char*>(w->stage);
     w->d_coords = reinterpret_cast<int32_t*>(base);
     w->d_res = w->d_coords + 3 * n;
@@ -308,8 +307,8 @@ int build_batch(uw_world* w, int32_t k, const Key& sc) {
     if (tot.n_inds > 0) {
         const uw_mesh_sections s = uw_sections(tot.n_verts, tot.n_inds, format_of(w->cfg));
         size_t bytes = 0;
-        void* block = uw_block_take(ctx, s.total, &bytes);  // (the device is idle: no one reads the block)
-        if (!block) return uw_fail(ctx, UW_ERR_HIP, "no device memory for a world arena");
+        void* block = nullptr;  // (the device is idle: no one reads the block)
+        if (int rc = uw_block_take(ctx, s.total, &block, &bytes)) return rc;
         if (!w->free_arenas.empty()) {
             arena = w->free_arenas.back();
             w->free_arenas.pop_back();
