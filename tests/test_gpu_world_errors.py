@@ -32,3 +32,34 @@ def test_no_memory_for_a_batch_is_out_of_memory():
         torch.cuda.synchronize()
         assert all(np.array_equal(x, y) for x, y in zip(before.chunk_mesh(0), after.chunk_mesh(0)))
     world.close()
+
+
+def _unfit(perlin):
+    """A launch shape whose workgroup fits no compute unit (33^3 densities in LDS)."""
+    from underwaterworld_amd import get_batch_tuning
+    return dict(get_batch_tuning(perlin), bulk_min=0, max_res=32, block=512, slab=[1] + list(range(1, 33)))
+
+
+def test_reported_error_does_not_reach_later_calls():
+    # a batched build that HIP refuses, then calls that launch kernels of their own
+    import torch
+    from underwaterworld_amd import Chunk, Perlin, _lib, build_chunks_batched, get_batch_tuning, set_batch_tuning
+    from underwaterworld_amd.world import World
+    perlin = Perlin(PR.preset("reference"))
+    good = get_batch_tuning(perlin)
+    world = World(perlin)
+    assert _step(world, [5.0, 7.0, -3.0]) > 0
+    where = world.chunks_to_render()[0]
+    want = world.get_chunk(where)
+    for _ in range(2):
+        set_batch_tuning(perlin, _unfit(perlin))
+        with pytest.raises(_lib.UwError):
+            build_chunks_batched(perlin, [where], 12)
+        set_batch_tuning(perlin, good)
+        got = world.get_chunk(where)
+        assert np.array_equal(got.verts, want.verts) and np.array_equal(got.inds, want.inds)
+    chunk = Chunk(where, resolution=12)
+    chunk.build_full(perlin)
+    assert np.array_equal(chunk.verts_buffer_slice(), want.verts)
+    torch.cuda.synchronize()
+    world.close()

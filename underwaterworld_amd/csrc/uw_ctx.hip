@@ -15,6 +15,7 @@ int uw_fail(uw_ctx* ctx, int code, const std::string& msg) {
 }
 
 int uw_hip_fail(uw_ctx* ctx, hipError_t e, const char* what) {
+    (void)hipGetLastError();  // reported here; left behind, the check after the next call's launches would find it
     std::string m = std::string(what) + ": " + hipGetErrorString(e);
     return uw_fail(ctx, e == hipErrorOutOfMemory ? UW_ERR_OOM : UW_ERR_HIP, m);
 }

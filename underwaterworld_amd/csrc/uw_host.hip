@@ -125,7 +125,6 @@ int uw_block_take(uw_ctx* ctx, size_t bytes, void** out, size_t* got) {
     }
     const hipError_t e = hipMalloc(out, bytes);
     if (e == hipSuccess) return UW_OK;
-    (void)hipGetLastError();  // reported here, not by the next launch
     *out = nullptr;
     *got = 0;
     return uw_hip_fail(ctx, e, "hipMalloc");
