@@ -63,3 +63,35 @@ def test_reported_error_does_not_reach_later_calls():
     assert np.array_equal(chunk.verts_buffer_slice(), want.verts)
     torch.cuda.synchronize()
     world.close()
+
+
+def test_failed_update_gives_the_buffer_back():
+    # a launch shape that HIP refuses: the update fails after its coordinates are on their way through the
+    # page-locked buffer. The next holder of the buffer, another world or the same one with its
+    # shape back, gets and gives its own data
+    from underwaterworld_amd import Perlin, _lib, get_batch_tuning, set_batch_tuning
+    from underwaterworld_amd.world import World
+    perlin = Perlin(PR.preset("reference"))
+    good = get_batch_tuning(perlin)
+    world, other, fresh = World(perlin), World(perlin), World(perlin)
+    assert _step(fresh, [5.0, 7.0, -3.0]) > 0 and _step(other, [400.0, -90.0, -3.0]) > 0
+    where = [c for c in fresh.chunks_to_render()[:8]]
+    there = [c for c in other.chunks_to_render()[:8]]
+    want, keep = [fresh.get_chunk(c) for c in where], [other.get_chunk(c) for c in there]
+    assert len(where) == 8 and len(there) == 8
+    for _ in range(4):
+        set_batch_tuning(perlin, _unfit(perlin))
+        with pytest.raises(_lib.UwError):
+            _step(world, [5.0, 7.0, -3.0])
+        assert world.total_count() == 0
+        for c, k in zip(there, keep):
+            g = other.get_chunk(c)
+            assert np.array_equal(g.verts, k.verts) and np.array_equal(g.inds, k.inds)
+        set_batch_tuning(perlin, good)
+    assert _step(world, [5.0, 7.0, -3.0]) > 0
+    for c, w in zip(where, want):
+        g = world.get_chunk(c)
+        assert np.array_equal(g.verts, w.verts) and np.array_equal(g.inds, w.inds)
+        assert np.array_equal(g.tri_cells, w.tri_cells) and np.array_equal(g.normals, w.normals)
+    for w in (world, other, fresh):
+        w.close()

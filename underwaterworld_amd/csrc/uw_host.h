@@ -38,8 +38,19 @@ __host__ __device__ inline uw_mesh_sections uw_sections(uint64_t nv, uint64_t ni
     return s;
 }
 
+// Holds ctx->host_lock while a call uses the page-locked buffer. Kernels on the null stream read and write
+// the buffer: a call that leaves before it has waited for them (an error) waits here, before the lock is
+// given up and the next holder writes the buffer, or grows it.
+struct uw_pinned_use {
+    std::unique_lock<std::mutex> lock;
+    bool pending = false;  // a kernel that uses the buffer may still run
+    explicit uw_pinned_use(uw_ctx* ctx) : lock(ctx->host_lock) {}
+    ~uw_pinned_use() {
+        if (pending) (void)hipStreamSynchronize(nullptr);
+    }
+};
 // The context's page-locked buffer with room for `bytes`, kept and grown to at most 16 MiB; false where
-// it can't be had (the caller copies directly). The caller holds ctx->host_lock while it uses the buffer.
+// it can't be had (the caller copies directly). The caller holds a uw_pinned_use while it uses the buffer.
 bool uw_pinned(uw_ctx* ctx, size_t bytes, unsigned char** p);
 int uw_copy_launch(uw_ctx* ctx, const uw_copies& c, hipStream_t st);
 int uw_chunk_out_launch(uw_ctx* ctx, const uw_chunk_info* info, const uw_mesh_ptrs& m, const uw_mesh_format& f,

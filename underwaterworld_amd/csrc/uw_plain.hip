@@ -792,13 +792,15 @@ int uw_chunk_build_host_out(uw_ctx* ctx, int32_t cx, int32_t cy, int32_t cz, int
     const size_t vfl = ho->vertex_format == UW_VERTEX_XYZ_RGB ? 6 : 3;
     const size_t isz = ho->index_format == UW_INDEX_U16 ? sizeof(uint16_t) : sizeof(uint32_t);
     {  // the record and the arrays together, if they fit
-        std::lock_guard<std::mutex> lock(ctx->host_lock);
+        uw_pinned_use use(ctx);
         unsigned char* pin;
         if (uw_pinned(ctx, kChunkPinned, &pin)) {
             const uw_mesh_ptrs m = {{ctx->d_verts1, ctx->d_inds1, ctx->d_norm1, ctx->d_cells1}};
             const uw_mesh_format f = {uint32_t(vfl * sizeof(float)), uint32_t(isz), want_norm ? 1u : 0u, want_cells ? 1u : 0u};
+            use.pending = true;
             if (int rc = uw_chunk_out_launch(ctx, ctx->d_info1, m, f, pin, kChunkPinned, nullptr)) return rc;
             UW_HIP(ctx, hipStreamSynchronize(nullptr));
+            use.pending = false;
             memcpy(info, pin, sizeof(*info));
             if (info->n_verts > ho->vert_cap || info->n_inds > ho->ind_cap)
                 return uw_fail(ctx, UW_ERR_OVERFLOW, "output capacity too small for this chunk");

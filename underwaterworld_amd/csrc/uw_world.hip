@@ -275,7 +275,7 @@ int build_batch(uw_world* w, int32_t k, const Key& sc) {
     std::vector<uw_chunk_info> info(static_cast<size_t>(k));
     uw_totals tot;
     {
-        std::lock_guard<std::mutex> lock(ctx->host_lock);
+        uw_pinned_use use(ctx);
         unsigned char* pin;
         const size_t in_room = (in_bytes + 255) & ~size_t(255);
         const bool pinned = uw_pinned(ctx, in_room + out_bytes, &pin);
@@ -283,6 +283,7 @@ int build_batch(uw_world* w, int32_t k, const Key& sc) {
             memcpy(pin, input.data(), in_bytes);
             const uw_copies c = {{pin, pin + size_t(k) * 12, nullptr, nullptr}, {w->d_coords, w->d_res, nullptr, nullptr},
                                  {uint64_t(k) * 12, uint64_t(k) * 4, 0, 0}};
+            use.pending = true;
             if (int rc = uw_copy_launch(ctx, c, nullptr)) return rc;
         } else {
             UW_HIP(ctx, hipMemcpy(w->d_coords, input.data(), size_t(k) * 12, hipMemcpyHostToDevice));
@@ -294,6 +295,7 @@ int build_batch(uw_world* w, int32_t k, const Key& sc) {
             if (int rc = uw_copy_launch(ctx, c, nullptr)) return rc;
         }
         UW_HIP(ctx, hipDeviceSynchronize());
+        use.pending = false;
         if (pinned) {
             memcpy(&tot, pin + in_room, sizeof(tot));
             memcpy(info.data(), pin + in_room + sizeof(tot), info.size() * sizeof(uw_chunk_info));
@@ -502,7 +504,7 @@ int uw_world_read_chunk(const uw_world* w, int32_t x, int32_t y, int32_t z, cons
         const uw_mesh_format f = {ho->verts ? uint32_t(vert_bytes(w->cfg)) : 0u, ho->inds ? uint32_t(ind_bytes(w->cfg)) : 0u,
                                   norm ? 1u : 0u, cells ? 1u : 0u};
         const uw_mesh_sections s = uw_sections(c.info.n_verts, c.info.n_inds, f);
-        std::lock_guard<std::mutex> lock(ctx->host_lock);
+        uw_pinned_use use(ctx);
         unsigned char* pin;
         if (uw_pinned(ctx, s.total, &pin)) {
             uw_copies p = {{c.verts, c.inds, c.tri_normals, c.tri_cells}, {}, {}};
@@ -511,8 +513,10 @@ int uw_world_read_chunk(const uw_world* w, int32_t x, int32_t y, int32_t z, cons
                 p.dst[k] = pin + s.off[k];
                 p.bytes[k] = s.bytes[k];
             }
+            use.pending = true;
             if (int rc = uw_copy_launch(ctx, p, nullptr)) return rc;
             UW_HIP(ctx, hipStreamSynchronize(nullptr));
+            use.pending = false;
             for (int k = 0; k < 4; ++k)
                 if (s.bytes[k]) memcpy(dst[k], pin + s.off[k], s.bytes[k]);
             return UW_OK;
