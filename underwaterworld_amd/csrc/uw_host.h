@@ -57,10 +57,11 @@ int uw_chunk_out_launch(uw_ctx* ctx, const uw_chunk_info* info, const uw_mesh_pt
                         unsigned char* dst, uint64_t cap, hipStream_t st);
 int uw_set_coord_launch(uw_ctx* ctx, int32_t* d_coord, int32_t x, int32_t y, int32_t z, hipStream_t st);
 
-// Device blocks kept by the context between uses (freed with it): at most kBlocksMax bytes and
-// kBlocksCount blocks, the rest is freed at once. A block may still be read by work queued before it was
-// given back: a taker synchronises the device after the take and before it writes.
-constexpr size_t kBlocksMax = size_t(256) << 20, kBlocksCount = 64;
+// Device blocks kept by the context between uses (uw_blocks.h; freed with it). A block may still be read
+// by work queued before it was given back: a taker synchronises the device after the take and before it
+// writes.
 int uw_block_take(uw_ctx* ctx, size_t bytes, void** out, size_t* got);
 void uw_block_give(uw_ctx* ctx, void* p, size_t bytes);
+// Frees the kept blocks; whether there were any.
+bool uw_blocks_release(uw_ctx* ctx);
 void uw_host_release(uw_ctx* ctx);

@@ -97,17 +97,11 @@ int uw_set_coord_launch(uw_ctx* ctx, int32_t* d_coord, int32_t x, int32_t y, int
 }
 
 int uw_block_take(uw_ctx* ctx, size_t bytes, void** out, size_t* got) {
+    bytes = uw_block_pool::rounded(bytes);
     {
-        std::lock_guard<std::mutex> lock(ctx->host_lock);
-        size_t best = ctx->blocks.size();
-        for (size_t i = 0; i < ctx->blocks.size(); ++i)
-            if (ctx->blocks[i].bytes >= bytes && ctx->blocks[i].bytes / 4 <= bytes &&
-                (best == ctx->blocks.size() || ctx->blocks[i].bytes < ctx->blocks[best].bytes))
-                best = i;
-        if (best < ctx->blocks.size()) {
-            const uw_block b = ctx->blocks[best];
-            ctx->blocks.erase(ctx->blocks.begin() + std::ptrdiff_t(best));
-            ctx->blocks_bytes -= b.bytes;
+        std::lock_guard<std::mutex> lock(ctx->blocks_lock);
+        uw_block b;
+        if (ctx->blocks.take(bytes, &b)) {
             *got = b.bytes;
             *out = b.p;
             return UW_OK;
@@ -117,12 +111,7 @@ int uw_block_take(uw_ctx* ctx, size_t bytes, void** out, size_t* got) {
     *got = bytes;
     if (hipMalloc(out, bytes) == hipSuccess) return UW_OK;
     (void)hipGetLastError();
-    {  // the kept blocks may be what is missing
-        std::lock_guard<std::mutex> lock(ctx->host_lock);
-        for (const uw_block& b : ctx->blocks) (void)hipFree(b.p);
-        ctx->blocks.clear();
-        ctx->blocks_bytes = 0;
-    }
+    uw_blocks_release(ctx);  // the kept blocks may be what is missing
     const hipError_t e = hipMalloc(out, bytes);
     if (e == hipSuccess) return UW_OK;
     *out = nullptr;
@@ -132,21 +121,17 @@ int uw_block_take(uw_ctx* ctx, size_t bytes, void** out, size_t* got) {
 
 void uw_block_give(uw_ctx* ctx, void* p, size_t bytes) {
     if (!p) return;
-    {
-        std::lock_guard<std::mutex> lock(ctx->host_lock);
-        if (ctx->blocks_bytes + bytes <= kBlocksMax && ctx->blocks.size() < kBlocksCount) {
-            ctx->blocks.push_back(uw_block{p, bytes});
-            ctx->blocks_bytes += bytes;
-            return;
-        }
-    }
-    (void)hipFree(p);
+    std::lock_guard<std::mutex> lock(ctx->blocks_lock);
+    ctx->blocks.give(uw_block{p, bytes}, [](const uw_block& b) { (void)hipFree(b.p); });
+}
+
+bool uw_blocks_release(uw_ctx* ctx) {
+    std::lock_guard<std::mutex> lock(ctx->blocks_lock);
+    return ctx->blocks.clear([](const uw_block& b) { (void)hipFree(b.p); });
 }
 
 void uw_host_release(uw_ctx* ctx) {
-    for (const uw_block& b : ctx->blocks) (void)hipFree(b.p);
-    ctx->blocks.clear();
-    ctx->blocks_bytes = 0;
+    uw_blocks_release(ctx);
     if (ctx->h_pinned) (void)hipHostFree(ctx->h_pinned);
     ctx->h_pinned = nullptr;
     ctx->pinned_bytes = 0;

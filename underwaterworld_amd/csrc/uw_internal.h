@@ -10,6 +10,7 @@
 
 #include "../../include/uwmesh.h"
 #include "mc_table.h"
+#include "uw_blocks.h"
 #include "uw_div.h"
 
 // Device-resident lookup tables, uploaded once per context.
@@ -61,12 +62,6 @@ struct uw_occupancy {
     int per_cu;
 };
 
-// A device block kept by a context between uses (uw_host.h).
-struct uw_block {
-    void* p;
-    size_t bytes;
-};
-
 struct uw_ctx {
     uw_params params;
     int device = 0;
@@ -110,12 +105,12 @@ struct uw_ctx {
     uint64_t verts1_cap = 0, inds1_cap = 0;
     uw_occupancy occupancy[64] = {};  // the last launch shapes seen (uw_resident), in a ring
     uint32_t occupancy_next = 0;
-    // host transfers (uw_host.h): the page-locked buffer and the kept blocks, under host_lock
+    // host transfers (uw_host.h): the page-locked buffer and the kept blocks, each under its lock
     std::mutex host_lock;
     unsigned char* h_pinned = nullptr;
     size_t pinned_bytes = 0;
-    std::vector<uw_block> blocks;
-    size_t blocks_bytes = 0;
+    std::mutex blocks_lock;
+    uw_block_pool blocks;
     std::string last_error;
 };
 
