@@ -328,7 +328,7 @@ int ensure_buffer(uw_ctx* ctx, void** buf, size_t* have, size_t bytes) {
     (void)hipFree(*buf);
     *buf = nullptr;
     *have = 0;
-    UW_HIP(ctx, hipMalloc(buf, bytes));
+    UW_ALLOC(ctx, *buf, bytes);
     *have = bytes;
     return UW_OK;
 }

@@ -1149,29 +1149,29 @@ int prepare_batched(uw_ctx* ctx, int32_t nchunks, const uw_mesh_out* out, BatchL
         (void)hipFree(ctx->d_batch_order);
         ctx->d_batch_order = nullptr;
         ctx->batch_order_cap = 0;
-        UW_HIP(ctx, hipMalloc(&ctx->d_batch_order, order_bufs(nchunks).bytes));
+        UW_ALLOC(ctx, ctx->d_batch_order, order_bufs(nchunks).bytes);
         ctx->batch_order_cap = size_t(nchunks);
     }
-    if (!ctx->d_batch_head) UW_HIP(ctx, hipMalloc(&ctx->d_batch_head, kQueueBytes));
+    if (!ctx->d_batch_head) UW_ALLOC(ctx, ctx->d_batch_head, kQueueBytes);
     if (bl->ztab_bytes > ctx->batch_ztab_bytes) {
         (void)hipFree(ctx->d_batch_ztab);
         ctx->d_batch_ztab = nullptr;
         ctx->batch_ztab_bytes = 0;
-        UW_HIP(ctx, hipMalloc(&ctx->d_batch_ztab, bl->ztab_bytes));
+        UW_ALLOC(ctx, ctx->d_batch_ztab, bl->ztab_bytes);
         ctx->batch_ztab_bytes = bl->ztab_bytes;
     }
     if (bl->dscr_bytes > ctx->batch_dscr_bytes) {
         (void)hipFree(ctx->d_batch_dscr);
         ctx->d_batch_dscr = nullptr;
         ctx->batch_dscr_bytes = 0;
-        UW_HIP(ctx, hipMalloc(&ctx->d_batch_dscr, bl->dscr_bytes));
+        UW_ALLOC(ctx, ctx->d_batch_dscr, bl->dscr_bytes);
         ctx->batch_dscr_bytes = bl->dscr_bytes;
     }
     if (bl->bulk.bytes > ctx->batch_bulk_bytes) {
         (void)hipFree(ctx->d_batch_bulk);
         ctx->d_batch_bulk = nullptr;
         ctx->batch_bulk_bytes = 0;
-        UW_HIP(ctx, hipMalloc(&ctx->d_batch_bulk, bl->bulk.bytes));
+        UW_ALLOC(ctx, ctx->d_batch_bulk, bl->bulk.bytes);
         ctx->batch_bulk_bytes = bl->bulk.bytes;
     }
     return UW_OK;
@@ -1344,7 +1344,7 @@ int uw_batched_graph_create(uw_ctx* ctx, const int32_t* coords, const int32_t* r
     const size_t ord_bytes = (kQueueBytes + order_bufs(nchunks).bytes + 255) & ~size_t(255);
     const size_t ztab_bytes = (bl.ztab_bytes + 255) & ~size_t(255);
     const size_t dscr_bytes = (bl.dscr_bytes + 255) & ~size_t(255);
-    UW_HIP(ctx, hipMalloc(&gbuf, ord_bytes + ztab_bytes + dscr_bytes + bl.bulk.bytes));
+    UW_ALLOC(ctx, gbuf, ord_bytes + ztab_bytes + dscr_bytes + bl.bulk.bytes);
     unsigned char* gtasks = reinterpret_cast<unsigned char*>(gbuf) + kQueueBytes;
     unsigned char* gztab = reinterpret_cast<unsigned char*>(gbuf) + ord_bytes;
     float* gdscr = reinterpret_cast<float*>(gztab + ztab_bytes);

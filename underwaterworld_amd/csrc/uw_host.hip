@@ -96,6 +96,17 @@ int uw_set_coord_launch(uw_ctx* ctx, int32_t* d_coord, int32_t x, int32_t y, int
     return UW_OK;
 }
 
+int uw_device_alloc(uw_ctx* ctx, void** p, size_t bytes) {
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipErrorOutOfMemory && uw_blocks_release(ctx)) {
+        (void)hipGetLastError();
+        e = hipMalloc(p, bytes);
+    }
+    if (e == hipSuccess) return UW_OK;
+    *p = nullptr;
+    return uw_hip_fail(ctx, e, "hipMalloc");
+}
+
 int uw_block_take(uw_ctx* ctx, size_t bytes, void** out, size_t* got) {
     bytes = uw_block_pool::rounded(bytes);
     {
@@ -107,16 +118,9 @@ int uw_block_take(uw_ctx* ctx, size_t bytes, void** out, size_t* got) {
             return UW_OK;
         }
     }
-    *out = nullptr;
-    *got = bytes;
-    if (hipMalloc(out, bytes) == hipSuccess) return UW_OK;
-    (void)hipGetLastError();
-    uw_blocks_release(ctx);  // the kept blocks may be what is missing
-    const hipError_t e = hipMalloc(out, bytes);
-    if (e == hipSuccess) return UW_OK;
-    *out = nullptr;
-    *got = 0;
-    return uw_hip_fail(ctx, e, "hipMalloc");
+    const int rc = uw_device_alloc(ctx, out, bytes);
+    *got = rc == UW_OK ? bytes : 0;
+    return rc;
 }
 
 void uw_block_give(uw_ctx* ctx, void* p, size_t bytes) {

@@ -132,6 +132,14 @@ int uw_hip_fail(uw_ctx* ctx, hipError_t e, const char* what);
 constexpr size_t kDefaultLds = size_t(48) << 10;
 int uw_resident(uw_ctx* ctx, const void* kernel, int block, size_t lds, int* per_cu);
 
+// Device memory of the context. Where it is short, the blocks that the context keeps between uses are
+// freed first: what fits without them still fits.
+int uw_device_alloc(uw_ctx* ctx, void** p, size_t bytes);
+#define UW_ALLOC(ctx, ptr, bytes)                                                             \
+    do {                                                                                      \
+        if (int uw_rc_ = uw_device_alloc(ctx, reinterpret_cast<void**>(&(ptr)), bytes)) return uw_rc_; \
+    } while (0)
+
 #define UW_HIP(ctx, expr)                                        \
     do {                                                         \
         hipError_t _e = (expr);                                  \

@@ -587,7 +587,7 @@ int plain_args(uw_ctx* ctx, const int32_t* coords, int32_t nchunks, int32_t n, i
         (void)hipFree(ctx->d_plain);
         ctx->d_plain = nullptr;
         ctx->plain_bytes = 0;
-        UW_HIP(ctx, hipMalloc(&ctx->d_plain, lay->bytes));
+        UW_ALLOC(ctx, ctx->d_plain, lay->bytes);
         ctx->plain_bytes = lay->bytes;
     }
     unsigned char* base = ctx->d_plain;
@@ -762,9 +762,9 @@ int uw_chunk_build_host_out(uw_ctx* ctx, int32_t cx, int32_t cy, int32_t cz, int
     UW_HIP(ctx, hipSetDevice(ctx->device));
     const uint64_t vmax = uw_max_verts(n), imax = uw_max_inds(n);
     if (!ctx->d_coord1) {
-        UW_HIP(ctx, hipMalloc(&ctx->d_coord1, 3 * sizeof(int32_t)));
-        UW_HIP(ctx, hipMalloc(&ctx->d_info1, sizeof(uw_chunk_info)));
-        UW_HIP(ctx, hipMalloc(&ctx->d_totals1, sizeof(uw_totals)));
+        UW_ALLOC(ctx, ctx->d_coord1, 3 * sizeof(int32_t));
+        UW_ALLOC(ctx, ctx->d_info1, sizeof(uw_chunk_info));
+        UW_ALLOC(ctx, ctx->d_totals1, sizeof(uw_totals));
     }
     if (ctx->verts1_cap < vmax || ctx->inds1_cap < imax) {
         (void)hipFree(ctx->d_verts1);
@@ -776,14 +776,14 @@ int uw_chunk_build_host_out(uw_ctx* ctx, int32_t cx, int32_t cy, int32_t cz, int
         ctx->d_norm1 = nullptr;
         ctx->d_cells1 = nullptr;
         ctx->verts1_cap = ctx->inds1_cap = 0;
-        UW_HIP(ctx, hipMalloc(&ctx->d_verts1, vmax * 6 * sizeof(float)));
-        UW_HIP(ctx, hipMalloc(&ctx->d_inds1, imax * sizeof(uint32_t)));
+        UW_ALLOC(ctx, ctx->d_verts1, vmax * 6 * sizeof(float));
+        UW_ALLOC(ctx, ctx->d_inds1, imax * sizeof(uint32_t));
         ctx->verts1_cap = vmax;
         ctx->inds1_cap = imax;
     }
     const bool want_norm = ho->tri_normals != nullptr, want_cells = ho->tri_cells != nullptr;
-    if (want_norm && !ctx->d_norm1) UW_HIP(ctx, hipMalloc(&ctx->d_norm1, ctx->inds1_cap * sizeof(float)));
-    if (want_cells && !ctx->d_cells1) UW_HIP(ctx, hipMalloc(&ctx->d_cells1, ctx->inds1_cap / 3 * sizeof(uint32_t)));
+    if (want_norm && !ctx->d_norm1) UW_ALLOC(ctx, ctx->d_norm1, ctx->inds1_cap * sizeof(float));
+    if (want_cells && !ctx->d_cells1) UW_ALLOC(ctx, ctx->d_cells1, ctx->inds1_cap / 3 * sizeof(uint32_t));
     if (int rc = uw_set_coord_launch(ctx, ctx->d_coord1, cx, cy, cz, nullptr)) return rc;
     uw_mesh_out out = {ctx->d_verts1, ctx->d_inds1, ctx->d_info1, ctx->d_totals1, ctx->verts1_cap, ctx->inds1_cap,
                        ho->vertex_format, ho->index_format, want_norm ? ctx->d_norm1 : nullptr,

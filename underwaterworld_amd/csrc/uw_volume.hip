@@ -588,7 +588,7 @@ int vol_prepare(uw_ctx* ctx, int32_t cx, int32_t cy, int32_t cz, int32_t n, VolA
         (void)hipFree(ctx->d_vol);
         ctx->d_vol = nullptr;
         ctx->vol_bytes = 0;
-        UW_HIP(ctx, hipMalloc(&ctx->d_vol, lay->bytes));
+        UW_ALLOC(ctx, ctx->d_vol, lay->bytes);
         ctx->vol_bytes = lay->bytes;
     }
     unsigned char* base = ctx->d_vol;
