@@ -58,3 +58,37 @@ def test_kept_blocks_make_room():
         torch.cuda.synchronize()
     v, ix = few.chunk_mesh(0)
     assert np.array_equal(verts[:len(v)].cpu().numpy(), v) and np.array_equal(inds[:len(ix)].cpu().numpy().view(np.uint32), ix)
+
+
+@pytest.mark.parametrize("octaves,n,count,left", [(4, 12, 8192, 64), (6, 24, 3000, 400)])
+def test_batched_without_room_for_the_bulk_scratch(octaves, n, count, left):
+    # scratch of about 110 and 480 MB that the bulk path would take; the persistent kernel needs none for
+    # chunks built in one pass and about 150 MB for those in x-slabs. Graphs own theirs, in the same way
+    import torch
+    from underwaterworld_amd import BatchedGraph, Perlin, build_chunks_batched
+    perlin = Perlin(PR.preset("chunks12" if octaves == 4 else "mixed", octaves=octaves))
+    coords = torch.as_tensor(np.tile(np.int32([[0, 0, 9]]), (count, 1)), device="cuda")
+    coords[:4] = torch.tensor([[0, 0, -1], [3, 1, -1], [0, 0, 0], [1, 2, 0]], dtype=torch.int32)
+    res = torch.full((count,), n, dtype=torch.int32, device="cuda")
+    few = build_chunks_batched(Perlin(perlin.params), coords[:4], n)
+    caps = dict(vert_cap=60000, ind_cap=200000)
+    other = Perlin(perlin.params, apply_tuning=False)
+    from test_gpu_bulk import _set_bulk
+    _set_bulk(other, 0)  # (the persistent kernel is loaded while there is memory)
+    build_chunks_batched(other, coords[:4], n)
+    torch.cuda.synchronize()
+    with _memory_left(left):
+        b = build_chunks_batched(perlin, coords, res, **caps)
+        g = BatchedGraph(perlin, coords, res, **caps)
+        gb = g.launch()
+        torch.cuda.synchronize()
+    again = build_chunks_batched(perlin, coords, res, **caps)
+    torch.cuda.synchronize()
+    want = few.info()
+    for got in (b, gb, again):
+        info = got.info()
+        assert got.totals()["overflow"] == 0 and not info["n_inds"][4:].any()
+        for i in range(4):
+            assert tuple(info[i])[:4] == tuple(want[i])[:4]
+            assert all(np.array_equal(x, y) for x, y in zip(got.chunk_mesh(i, info), few.chunk_mesh(i, want)))
+    g.close()

@@ -41,8 +41,8 @@ constexpr int kDensBudget = 20 * 1024;  // default LDS bytes for the density sla
 // over the device, the persistent kernel holds a whole chunk in one workgroup): 41 us of kernels against
 // 75 for a world update, 98 against 196 for 1000 chunks of 3 .. 32 cells, 517 against 577 for 8192 of
 // 8 .. 32, a launch of 4096 of 12^3 at 3 octaves 91 against 121. The persistent kernel is left with
-// launches of few small chunks (few_small), those whose bulk scratch would pass its limit, and a larger
-// bulk_min set by the caller.
+// launches of few small chunks (few_small), those whose bulk scratch would pass its limit or can't be had,
+// and a larger bulk_min set by the caller.
 constexpr int kDefaultBulkMin = 1;
 
 struct BatchArgs {
@@ -1142,9 +1142,21 @@ int shape_batched(uw_ctx* ctx, int32_t nchunks, bool extra, BatchLaunch* bl, boo
     return UW_OK;
 }
 
-// shape_batched plus the context-owned scratch of the eager path (grown as needed).
+// shape_batched plus the context-owned scratch of the eager path (grown as needed). The bulk path's
+// scratch (up to 8 GiB) is the one part that a launch can do without: where it can't be had, the chunks
+// stay on the persistent kernel.
 int prepare_batched(uw_ctx* ctx, int32_t nchunks, const uw_mesh_out* out, BatchLaunch* bl) {
-    if (int rc = shape_batched(ctx, nchunks, uw_emit_extra(uw_make_emit_opts(out)), bl)) return rc;
+    const bool extra = uw_emit_extra(uw_make_emit_opts(out));
+    if (int rc = shape_batched(ctx, nchunks, extra, bl)) return rc;
+    if (bl->bulk.bytes > ctx->batch_bulk_bytes) {
+        (void)hipFree(ctx->d_batch_bulk);
+        ctx->d_batch_bulk = nullptr;
+        ctx->batch_bulk_bytes = 0;
+        const int rc = uw_device_alloc(ctx, reinterpret_cast<void**>(&ctx->d_batch_bulk), bl->bulk.bytes);
+        if (rc == UW_OK) ctx->batch_bulk_bytes = bl->bulk.bytes;
+        else if (rc != UW_ERR_OOM) return rc;
+        else if (int rc2 = shape_batched(ctx, nchunks, extra, bl, false)) return rc2;
+    }
     if (size_t(nchunks) > ctx->batch_order_cap) {
         (void)hipFree(ctx->d_batch_order);
         ctx->d_batch_order = nullptr;
@@ -1166,13 +1178,6 @@ int prepare_batched(uw_ctx* ctx, int32_t nchunks, const uw_mesh_out* out, BatchL
         ctx->batch_dscr_bytes = 0;
         UW_ALLOC(ctx, ctx->d_batch_dscr, bl->dscr_bytes);
         ctx->batch_dscr_bytes = bl->dscr_bytes;
-    }
-    if (bl->bulk.bytes > ctx->batch_bulk_bytes) {
-        (void)hipFree(ctx->d_batch_bulk);
-        ctx->d_batch_bulk = nullptr;
-        ctx->batch_bulk_bytes = 0;
-        UW_ALLOC(ctx, ctx->d_batch_bulk, bl->bulk.bytes);
-        ctx->batch_bulk_bytes = bl->bulk.bytes;
     }
     return UW_OK;
 }
@@ -1343,8 +1348,14 @@ int uw_batched_graph_create(uw_ctx* ctx, const int32_t* coords, const int32_t* r
     uint32_t* gbuf = nullptr;
     const size_t ord_bytes = (kQueueBytes + order_bufs(nchunks).bytes + 255) & ~size_t(255);
     const size_t ztab_bytes = (bl.ztab_bytes + 255) & ~size_t(255);
-    const size_t dscr_bytes = (bl.dscr_bytes + 255) & ~size_t(255);
-    UW_ALLOC(ctx, gbuf, ord_bytes + ztab_bytes + dscr_bytes + bl.bulk.bytes);
+    size_t dscr_bytes = 0;
+    for (;;) {
+        dscr_bytes = (bl.dscr_bytes + 255) & ~size_t(255);
+        const int rc = uw_device_alloc(ctx, reinterpret_cast<void**>(&gbuf), ord_bytes + ztab_bytes + dscr_bytes + bl.bulk.bytes);
+        if (rc == UW_OK) break;
+        if (rc != UW_ERR_OOM || !bl.bulk.on) return rc;
+        if (int rc2 = shape_batched(ctx, nchunks, false, &bl, false)) return rc2;  // (as prepare_batched)
+    }
     unsigned char* gtasks = reinterpret_cast<unsigned char*>(gbuf) + kQueueBytes;
     unsigned char* gztab = reinterpret_cast<unsigned char*>(gbuf) + ord_bytes;
     float* gdscr = reinterpret_cast<float*>(gztab + ztab_bytes);
