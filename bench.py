@@ -16,7 +16,7 @@ workload (8192 chunks, 25 % each at 8^3, 12^3, 24^3, 32^3, 6 octaves), the adjoi
 chunks of 24^3, forward + backward) and the single 512^3 volume (513^3 samples, 8 octaves,
 forward + adjoint with the noise recomputed in the backward) with its device-wide memory use.
 
-`roofline`: the density and row kernels of the headline path (its persistent kernel where it has one),
+`roofline`: the density kernel of the headline path (its persistent kernel where it has one),
 FP32-VALU bound, algorithmic FLOPs F(O) = 78 O + 6 per sample (per launch F(4) * 13^3 * 4096 =
 2.86 GFLOP), timed with HIP events recorded by the library on the launch stream around them. `cpu_baseline`: the reference CPU
 path (the oracle's reference-faithful C restatement: f64 noise, literal linear-search dedup), one
@@ -129,6 +129,14 @@ def main():
         L.uw_profile_enable(perlin.ctx, 0)
         return [tot[i] / cnt[i] if cnt[i] else None for i in range(k)]
 
+    def batched_stages(perlin, st):
+        """Named stages (ms) of a batched build: where every chunk takes the bulk path, stage 0 is its
+        density kernel and the front its row counts."""
+        bulk = st[_lib.STAGE_BULK_EMIT] is not None and get_batch_tuning(perlin)["bulk_min"] == 1
+        names = (("setup", _lib.STAGE_BATCH_SETUP), ("bulk_density" if bulk else "persistent", _lib.STAGE_DOMINANT),
+                 ("bulk_rows" if bulk else "bulk_front", _lib.STAGE_BULK_FRONT), ("bulk_emit", _lib.STAGE_BULK_EMIT))
+        return {name: round(st[i], 4) for name, i in names if st[i] is not None}
+
     def log(msg):
         print(msg, file=sys.stderr, flush=True)
 
@@ -233,11 +241,11 @@ def main():
         log(f"# plain path, one chunk per call: {ms_single * 1e3:.2f} us/chunk")
         st_b = stage_ms(perlin, batched_step, args.steps)
         st_p = stage_ms(perlin, plain_step, args.steps)
-        # a launch whose chunks all take the bulk path has no persistent kernel: its density and row kernels
-        persistent = st_b[_lib.STAGE_DOMINANT] is not None
-        ms_kernel = st_b[_lib.STAGE_DOMINANT if persistent else _lib.STAGE_BULK_FRONT]
+        # a launch whose chunks all take the bulk path has no persistent kernel: its density kernel instead
+        persistent = st_b[_lib.STAGE_BULK_EMIT] is None or get_batch_tuning(perlin)["bulk_min"] != 1
+        ms_kernel = st_b[_lib.STAGE_DOMINANT]
         ms_noise_plain = st_p[_lib.STAGE_DOMINANT]
-        kernel_name = "k_batched (persistent: density + mesh)" if persistent else "k_bulk_density + k_bulk_rows"
+        kernel_name = "k_batched (persistent: density + mesh)" if persistent else "k_bulk_density"
         path_name = "persistent kernel" if persistent else "bulk path"
         log(f"# {kernel_name} {ms_kernel:.4f} ms; plain stages {st_p[:4]}")
 
@@ -327,9 +335,7 @@ def main():
         # per-stage kernel times of the same build launched eagerly (a graph records no timers)
         st_m = stage_ms(pmix, lambda: build_chunks_batched(pmix, mc, mr, vert_cap=mv, ind_cap=mi,
                                                            stream=stream.cuda_stream), 3)
-        mixed_stages = {name: round(st_m[i], 4) for name, i in (
-            ("setup", _lib.STAGE_BATCH_SETUP), ("bulk_front", _lib.STAGE_BULK_FRONT),
-            ("persistent", _lib.STAGE_DOMINANT), ("bulk_emit", _lib.STAGE_BULK_EMIT)) if st_m[i] is not None}
+        mixed_stages = batched_stages(pmix, st_m)
         samples = int(sum((r + 1) ** 3 for r in mr))
         flops_m = flops_per_sample(pm["octaves"]) * samples
         res["mixed"] = {"workload": "8192 chunks, 2048 each at 8^3/12^3/24^3/32^3 cells, coords uniform in 32x32x8 "
@@ -364,11 +370,9 @@ def main():
         ms_adj = timed(adj_step, max(10, args.steps // 2), 2)
         st_f = stage_ms(pad, lambda: mesher.forward(stream.cuda_stream), 3)
         st_a = stage_ms(pad, lambda: mesher.backward(gv, stream.cuda_stream, record=rec), 3)
-        # the forward's launches: queue set-up, the bulk path's front and emission (24^3 chunks leave
-        # the persistent queue when the tuning's bulk_min allows) and the persistent kernel
-        fwd_stages = {name: round(st_f[i], 4) for name, i in (
-            ("setup", _lib.STAGE_BATCH_SETUP), ("bulk_front", _lib.STAGE_BULK_FRONT),
-            ("persistent", _lib.STAGE_DOMINANT), ("bulk_emit", _lib.STAGE_BULK_EMIT)) if st_f[i] is not None}
+        # the forward's launches: queue set-up, the bulk path (24^3 chunks leave the persistent queue when
+        # the tuning's bulk_min allows) and the persistent kernel where it has chunks left
+        fwd_stages = batched_stages(pad, st_f)
         fwd_ms = sum(fwd_stages.values())
         res["adjoint"] = {"workload": "256 chunks (x,y in [-4,4), z in [-3,1)) x 24^3 cells, 6 octaves, seed 42; "
                                       "forward with vertex tape + backward to 25^3 densities, 6 amplitudes, 3 offsets",

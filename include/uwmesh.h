@@ -144,9 +144,9 @@ void uw_permutation_table(uint32_t seed, uint8_t* out256);
 
 /* Kernel timing: while enabled, every build records HIP events on its stream around its kernels,
  * each pair tagged with a stage. Stage 0 is the path's dominant kernel: the density kernel of the
- * plain path, the persistent kernel of the batched path (absent from launches whose chunks all take
- * the bulk path), the density kernel of the volume path and the backward kernel(s) of the adjoint. uw_profile_read synchronises on the recorded events,
- * returns the summed milliseconds and the number of timed launches of stage 0 since the last read,
+ * plain path, the persistent kernel of the batched path (its bulk density kernel where every chunk takes
+ * the bulk path), the density kernel of the volume path and the backward kernel(s) of the adjoint.
+ * uw_profile_read synchronises on the recorded events, returns the summed milliseconds and the number of timed launches of stage 0 since the last read,
  * and resets every stage; uw_profile_read_stages does the same for stages [0, nstages) into
  * arrays. Not for use under graph capture. */
 enum uw_profile_stage {
@@ -159,7 +159,8 @@ enum uw_profile_stage {
     UW_STAGE_VOLUME_SCAN = 6,    /* k_vol_scan_* */
     UW_STAGE_VOLUME_EMIT = 7,    /* k_vol_emit */
     UW_STAGE_VOLUME_TABLES = 8,  /* k_vol_tables */
-    UW_STAGE_BULK_FRONT = 9,     /* k_bulk_density + k_bulk_rows (batched bulk path) */
+    UW_STAGE_BULK_FRONT = 9,     /* batched bulk path: k_bulk_density + k_bulk_rows, or k_bulk_rows alone where
+                                    the densities are stage 0 */
     UW_STAGE_BULK_EMIT = 10,     /* k_bulk_emit */
     UW_STAGE_COUNT = 11
 };

@@ -501,8 +501,13 @@ int uw_bulk_launch_front(uw_ctx* ctx, const uw_bulk_shape& s, const uw_bulk_io& 
     const BulkArgs a = bulk_args(ctx, s, io);
     const int block = bulk_density_block(s.max_res);
     const BulkDensityKernel kd = pick_bulk_density(ctx->params.octaves, block);
-    if (int rc = uw_prof_start(ctx, st, UW_STAGE_BULK_FRONT)) return rc;
+    // a launch of bulk chunks alone has its dominant kernel here, one with the persistent kernel has it there
+    if (int rc = uw_prof_start(ctx, st, io.all ? UW_STAGE_DOMINANT : UW_STAGE_BULK_FRONT)) return rc;
     hipLaunchKernelGGL(kd, dim3(uint32_t(s.grid_density)), dim3(uint32_t(block)), s.lds_density, st, a);
+    if (io.all) {
+        if (int rc = uw_prof_end(ctx, st)) return rc;
+        if (int rc = uw_prof_start(ctx, st, UW_STAGE_BULK_FRONT)) return rc;
+    }
     hipLaunchKernelGGL(s.rows_waves == 4 ? k_bulk_rows<4> : k_bulk_rows<16>, dim3(uint32_t(s.grid_rows)),
                        dim3(uint32_t(64 * s.rows_waves)), size_t(s.rows_waves) * size_t(s.max_tiles) * sizeof(uint32_t), st, a);
     if (int rc = uw_prof_end(ctx, st)) return rc;
