@@ -9,8 +9,9 @@ with 6 octaves, the 512^3 volume as 4096 bricks of 32^3 with 8 octaves) it times
             is built in one slab (one density evaluation); larger chunks use the largest x-slab
             that fits (densities evaluated twice)
     grid    persistent workgroups: all that fit (0)
-    bulk_min  chunks of at least this many cells per axis go to the bulk path (0: off); swept last
-            over the workload's resolutions
+    bulk_min  chunks of at least this many cells per axis go to the bulk path (0: off, 1: every chunk);
+            swept last, over the workload's resolutions. The shapes before it are timed with 0: a launch
+            whose chunks take the bulk path doesn't run the kernel that they shape
 with max_res set to the workload's largest resolution (it sizes the launch's LDS). The budget ties
 every resolution's x-slab size to one LDS figure; the fastest shape is then refined one x-slab
 resolution of the workload at a time (coordinate descent over that resolution's planes per slab,
@@ -122,14 +123,14 @@ def refine_slabs(perlin, coords, res, best_ms, best, steps, stream, ref, log=pri
 
 
 def refine_bulk(perlin, coords, res, best_ms, best, steps, stream, ref, log=print):
-    """The bulk path's threshold: off (0), or, for each distinct resolution r of the workload above
-    the one-pass sizes, one more than the largest resolution below r (chunks of at least bulk_min
-    cells per axis leave the persistent queue, whose LDS is then sized for bulk_min - 1: the
+    """The bulk path's threshold: off (0), every chunk (1), or, for each distinct resolution r of the
+    workload above the one-pass sizes, one more than the largest resolution below r (chunks of at least
+    bulk_min cells per axis leave the persistent queue, whose LDS is then sized for bulk_min - 1: the
     tightest threshold that moves r and above gives the persistent kernel its smallest shape)."""
     results = []
     rs = sorted({int(n) for n in res})
-    cands = [0] + [max([q for q in rs if q < r], default=0) + 1 for r in rs if 13 <= r <= int(best["max_res"])]
-    for b in cands:
+    cands = [0, 1] + [max([q for q in rs if q < r], default=0) + 1 for r in rs if 13 <= r <= int(best["max_res"])]
+    for b in dict.fromkeys(cands):
         if b == int(best.get("bulk_min", -1)):
             continue
         t = dict(best, slab=list(best["slab"]), bulk_min=b)
@@ -148,6 +149,7 @@ def tune_workload(perlin, coords, res, steps=10, quick=False, log=print, start=N
     from .engine import get_batch_tuning, set_batch_tuning
 
     base = get_batch_tuning(perlin)
+    off = dict(base, bulk_min=0)
     results = []
     ref = [None]
     stream = torch.cuda.current_stream()
@@ -157,7 +159,7 @@ def tune_workload(perlin, coords, res, steps=10, quick=False, log=print, start=N
         for block in blocks:
             for budget in budgets:
                 for grid in GRIDS:
-                    t = dict(base, block=block, grid=grid, max_res=int(max(res)), slab=slabs_for_budget(budget))
+                    t = dict(off, block=block, grid=grid, max_res=int(max(res)), slab=slabs_for_budget(budget))
                     ms = _time_shape(perlin, coords, res, t, steps, stream, ref, log,
                                      f"block={block} budget={budget} grid={grid}")
                     if ms is not None:
@@ -165,7 +167,7 @@ def tune_workload(perlin, coords, res, steps=10, quick=False, log=print, start=N
         results.sort(key=lambda r: r[0])
         best_ms, best = results[0]
     else:
-        best = dict(start, slab=list(start["slab"]))
+        best = dict(start, slab=list(start["slab"]), bulk_min=0)
         best_ms = _time_shape(perlin, coords, res, best, steps, stream, ref, log, "start")
         results.append((best_ms, best))
     best_ms, best, refined = refine_slabs(perlin, coords, res, best_ms, best, steps, stream, ref, log)
