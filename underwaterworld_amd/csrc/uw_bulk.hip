@@ -429,6 +429,8 @@ int uw_bulk_shape_for(uw_ctx* ctx, const uw_batch_tuning& t, int32_t nchunks, uw
         s->max_tiles = g.tiles > s->max_tiles ? g.tiles : s->max_tiles;
         rows = g.max_rows > rows ? g.max_rows : rows;
     }
+    if (!uw_emit_takes(rows, t.max_res, t.max_res))
+        return uw_fail(ctx, UW_ERR_INVALID_ARG, "emission tiles larger than a workgroup takes");
     s->lds_emit = uw_emit_lds_bytes(rows, t.max_res);
     const void* emit[2] = {reinterpret_cast<const void*>(k_bulk_emit<false>), reinterpret_cast<const void*>(k_bulk_emit<true>)};
     for (int extra = 0; extra < 2; ++extra)

@@ -700,6 +700,8 @@ int uw_build_chunks_plain(uw_ctx* ctx, const int32_t* coords, int32_t nchunks, i
         planes = (planes + 1) / 2;
         tiling = uw_tiling_for(n, planes);
     }
+    if (!uw_emit_takes(tiling.max_rows, tiling.cells + (tiling.yt > 1 ? 1 : 0), tiling.cells))
+        return uw_fail(ctx, UW_ERR_INVALID_ARG, "emission tiles larger than a workgroup takes");
     const uint64_t items = uint64_t(nchunks) * uint64_t(tiling.tiles());
     if (items > 0x7FFFFFFFull) return uw_fail(ctx, UW_ERR_INVALID_ARG, "too many chunks for one launch");
     PlainArgs a;

@@ -245,13 +245,14 @@ __device__ __forceinline__ unsigned long long uw_block_rows(const uint32_t* word
 // dense per-cell state, three workgroups a unit and the three corners of a triangle found one after the
 // other, took 1174 us there, 57 (now 36) for 150^3, 164 (now 122) for 8192 chunks of 8 .. 32 cells, 25 (now
 // 17) for 48 chunks of 48^3 and as much for 4096 of 12^3 (28). Fetching a tile's row segments a round ahead
-// was slower for chunks (147 where it was 141). A list of at most kListCap cells, whatever the tile, lets six
-// workgroups share a compute unit; a tile with more active cells (more than half of its cells, for 32
-// cells per axis) is emitted one plane at a time, which always fits.
+// was slower for chunks (147 where it was 141). A list of at most kListCap cells, whatever the tile, lets five
+// workgroups share a compute unit's 160 KB of LDS (29 KB each for tiles of 200 to 224 row segments), six for
+// tiles of up to 157 (27 KB); a tile with more active cells (more than half of its cells, for 32 cells per
+// axis) is emitted one plane at a time, which always fits.
 constexpr int kEmitThreads = 256;
 constexpr uint32_t kListCap = 2112;            // listed cells: two planes (one and its halo) of 33 rows of 32
 constexpr uint32_t kVertMap = 128, kTriMap = 192;  // map entries per wave
-constexpr int kEmitMaxRows = kEmitThreads;  // row segments of a tile, halo included
+constexpr int kEmitMaxRows = kEmitThreads;  // row segments of a tile, halo included: one thread each
 
 struct uw_emit_tile {
     uw_emit_opts eo;
@@ -275,6 +276,11 @@ static_assert(offsetof(uw_tables, before) == 2048 && offsetof(uw_tables, cell) =
 constexpr size_t kEmitWaveBytes = (kEmitThreads / 64) * (kVertMap + kTriMap) * 2;  // V2C, T2C
 __host__ __device__ constexpr uint32_t uw_emit_list_cap(int32_t rows, int32_t cells) {
     return uint32_t(rows) * uint32_t(cells) < kListCap ? uint32_t(rows) * uint32_t(cells) : kListCap;
+}
+// Whether the emitter takes tiles of `rows` row segments (halo included) of `cells` cells: a thread per row
+// segment, and a plane with its halo (at most two rows of `line` segments) always fits the list.
+__host__ __device__ constexpr bool uw_emit_takes(int32_t rows, int32_t line, int32_t cells) {
+    return rows <= kEmitMaxRows && 2u * uint32_t(line) * uint32_t(cells) <= kListCap;
 }
 // Bytes of dynamic LDS for tiles of `rows` row segments (halo included) of `cells` cells.
 __host__ __device__ constexpr size_t uw_emit_lds_bytes(int32_t rows, int32_t cells) {

@@ -724,6 +724,8 @@ int uw_build_volume(uw_ctx* ctx, int32_t cx, int32_t cy, int32_t cz, int32_t n, 
         planes = (planes + 1) / 2;
         a.tiling = uw_tiling_for(n, planes);
     }
+    if (!uw_emit_takes(a.tiling.max_rows, a.tiling.cells + (a.tiling.yt > 1 ? 1 : 0), a.tiling.cells))
+        return uw_fail(ctx, UW_ERR_INVALID_ARG, "emission tiles larger than a workgroup takes");
     const size_t elds = uw_emit_lds_bytes(a.tiling.max_rows, a.tiling.cells);
     using VolEmitKernel = void (*)(VolArgs);
     const VolEmitKernel ek = uw_emit_extra(a.eo) ? k_vol_emit<true> : k_vol_emit<false>;
