@@ -428,7 +428,7 @@ __device__ __forceinline__ void write_cases(const PlainArgs& a, uint32_t b) {
 // 12^3); else, for launches whose tiles all fit the device at once, workgroup b takes tile b, which
 // saves the look-ups. A chunk's first vertex and index are summed from the sizes before it (the groups
 // before its own, then the chunks of its group) by the workgroup itself, so no launch scans the chunks.
-template <bool LISTED, bool EXTRA>
+template <bool LISTED, bool EXTRA, bool CASES>
 __global__ void __launch_bounds__(kThreads, EXTRA ? 5 : 6) k_emit(PlainArgs a) {
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ unsigned long long s_sum[2][kThreads / 64];
@@ -436,12 +436,12 @@ __global__ void __launch_bounds__(kThreads, EXTRA ? 5 : 6) k_emit(PlainArgs a) {
         group_records(a, int32_t(blockIdx.x));
         return;
     }
-    if (int32_t(blockIdx.x) < a.ngroups + a.ncase) {
+    if (CASES && int32_t(blockIdx.x) < a.ngroups + a.ncase) {
         write_cases(a, blockIdx.x - uint32_t(a.ngroups));
         return;
     }
     const int tid = threadIdx.x;
-    const uint32_t before = uint32_t(a.ngroups) + uint32_t(a.ncase);
+    const uint32_t before = uint32_t(a.ngroups) + (CASES ? uint32_t(a.ncase) : 0u);
     const uint32_t tiles = uint32_t(a.tiling.tiles()), G = gridDim.x - before, b = blockIdx.x - before;
     uint32_t ends[kTileClasses], items = 0;  // listed tiles of the classes up to each
     if (LISTED) {
@@ -516,6 +516,11 @@ __global__ void __launch_bounds__(kThreads, EXTRA ? 5 : 6) k_emit(PlainArgs a) {
 }
 
 using EmitKernel = void (*)(PlainArgs);
+template <bool LISTED>
+EmitKernel pick_emit(bool extra, bool cases) {
+    if (cases) return extra ? k_emit<LISTED, true, true> : k_emit<LISTED, false, true>;
+    return extra ? k_emit<LISTED, true, false> : k_emit<LISTED, false, false>;
+}
 
 // Page-locked room for a host build's record and arrays (a full 12^3 chunk has 0.3 MB)
 constexpr uint64_t kChunkPinned = uint64_t(2) << 20;
@@ -717,7 +722,7 @@ int uw_build_chunks_plain(uw_ctx* ctx, const int32_t* coords, int32_t nchunks, i
     a.eo = uw_make_emit_opts(out);
     const size_t elds = uw_emit_lds_bytes(tiling.max_rows, tiling.cells);
     const bool extra = uw_emit_extra(a.eo);
-    const EmitKernel listed = extra ? k_emit<true, true> : k_emit<true, false>, all = extra ? k_emit<false, true> : k_emit<false, false>;
+    const EmitKernel listed = pick_emit<true>(extra, cases != nullptr), all = pick_emit<false>(extra, cases != nullptr);
     UW_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void*>(listed), hipFuncAttributeMaxDynamicSharedMemorySize, int(elds)));
     UW_HIP(ctx, hipFuncSetAttribute(reinterpret_cast<const void*>(all), hipFuncAttributeMaxDynamicSharedMemorySize, int(elds)));
     int per_cu = 0;
