@@ -591,5 +591,6 @@ __device__ __forceinline__ double uw_param_grad(const uw_field& f, const double*
     if (q < O) return (S[q] - S[O + 4] * inv_sum) * inv_sum;
     const double slope = f.bias_kind == UW_BIAS_LINEAR ? double(f.bias_a) : 0.0;
     const double g = S[q] * inv_sum;
-    return f.frequency * (q == O + 2 ? g + slope * S[O + 3] : g);
+    // (no slope, no term: 0 W would be NaN where a weight is infinite)
+    return f.frequency * (q == O + 2 && slope != 0.0 ? g + slope * S[O + 3] : g);
 }
