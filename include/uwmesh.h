@@ -227,7 +227,7 @@ int uw_chunk_build_host_out(uw_ctx* ctx, int32_t cx, int32_t cy, int32_t cz, int
 int uw_tris_around(const uint32_t* tri_cells, uint32_t ntris, int32_t n, float px, float py, float pz,
                    int32_t range, uint32_t* ids, uint32_t cap, uint32_t* count);
 
-/* ---- Batched path: one persistent launch over many chunks of mixed resolution ------------- */
+/* ---- Batched path: one call over many chunks of mixed resolution --------------------------- */
 
 #define UW_BATCH_MAX_RESOLUTION 32
 

@@ -197,7 +197,7 @@ private:
     std::vector<uint32_t> tri_cells_;
 };
 
-// A whole chunk set built by one persistent launch (uw_build_chunks_batched); results copied back
+// A whole chunk set built by one call (uw_build_chunks_batched); results copied back
 // to host memory per chunk. Device buffers are reused across builds of the same or smaller size.
 class ChunkBatch {
 public:

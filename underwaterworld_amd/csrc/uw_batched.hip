@@ -1,6 +1,8 @@
-// Batched path: thousands of chunks of mixed resolution meshed by ONE persistent launch.
+// Batched path: thousands of chunks of mixed resolution meshed in one call. The queue set-up and the
+// persistent kernel are here; the chunks of a launch go to the bulk path (uw_bulk.hip), to the persistent
+// kernel or, with a bulk_min between, to both (shape_batched).
 //
-// A fixed grid of workgroups (a few per CU) pulls chunk tasks from a global queue (atomic head
+// The persistent kernel. A fixed grid of workgroups (a few per CU) pulls chunk tasks from a global queue (atomic head
 // over a resolution-sorted order, largest chunks first). Each workgroup builds its chunk entirely
 // in LDS:
 //   1. per-axis octave tables of the chunk (uw_build_xy_tables, uw_ztab_block);
@@ -13,9 +15,9 @@
 //      lerps and the index writes. Vertex ids follow the reference's first-seen order through the
 //      edge-ownership rule (uw_mesh.h); each owner's vertex base and case sit in an LDS ring of the
 //      last cells.
-// Chunks that fit one slab compute their densities once; larger chunks recompute them in step 5
-// (the densities are not stored anywhere in HBM). The launch sequence (reset, order, persistent
-// kernel) has no host synchronisation, so it can be captured in a hipGraph.
+// Chunks that fit one slab compute their densities once; larger chunks reload them in step 5 from a
+// per-workgroup scratch, or recompute them where there is none (the no-allocation form). The launch
+// sequence has no host synchronisation, so it can be captured in a hipGraph.
 #include <hip/hip_runtime.h>
 #include <string.h>
 

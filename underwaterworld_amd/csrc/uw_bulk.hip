@@ -1,7 +1,6 @@
-// Bulk path of the batched build: chunks of at least `bulk_min` cells per axis (the 24^3 and 32^3
-// chunks of mixed-resolution and adjoint launches) leave the persistent queue. One workgroup per
-// chunk would run a 24^3 chunk's density, classification and emission as a serial chain of x-slab
-// phases; here every phase is spread over the device instead:
+// Bulk path of the batched build: chunks of at least `bulk_min` cells per axis (1, the default: all of
+// them) leave the persistent queue. One workgroup per chunk runs its density, classification and emission
+// as a serial chain; here every phase is spread over the device instead:
 //
 //   k_bulk_density  one lane per z-line (lanes on consecutive lines t = x L + y of one chunk),
 //                   densities into a per-chunk HBM field [z][t], so each sample's store is a row,

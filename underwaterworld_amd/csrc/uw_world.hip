@@ -4,7 +4,7 @@
 // the reference's f32 operation order (this file is compiled with -ffp-contract=off). The build
 // step differs by design: where the reference builds one chunk per frame (build_full_step /
 // build_step, world.rs:113-145), uw_world_update builds up to max_batch pending candidates in one
-// persistent launch (uw_build_chunks_batched) and then applies the reference's per-chunk rules to
+// call (uw_build_chunks_batched) and then applies the reference's per-chunk rules to
 // the results in pop order. Each launch's output is compacted into an arena of its size (one block, one
 // copy kernel); a chunk refers to its slice of an arena, and the arena's block goes back to the context
 // when its last chunk is evicted, as the launch staging does with the world.

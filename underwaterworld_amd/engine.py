@@ -367,7 +367,7 @@ def batch_capacity(res) -> tuple[int, int]:
 
 def build_chunks_batched(perlin: Perlin, coords, res, vert_cap: int | None = None, ind_cap: int | None = None,
                          stream=None, colors: bool = False, u16: bool = False, collision: bool = False) -> MeshBatch:
-    """One persistent launch over a mixed-resolution chunk set (res: cells per axis per chunk).
+    """One call over a mixed-resolution chunk set (res: cells per axis per chunk).
     colors=True writes the reference's VertColor layout (position + sRGB colour per vertex)."""
     import torch
     dev = torch.device("cuda", perlin.device)
