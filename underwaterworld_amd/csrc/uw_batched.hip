@@ -1414,12 +1414,13 @@ int uw_batched_graph_create(uw_ctx* ctx, const int32_t* coords, const int32_t* r
 namespace {
 constexpr size_t kNoAllocBytes = size_t(32) << 20;  // UW_NOALLOC_SCRATCH_BYTES
 constexpr int kNoAllocDevices = 64;
-static __device__ __align__(256) unsigned char scratch[kNoAllocBytes];
+// (the bulk path's counters at the end of the queue state aren't used here, and lie beyond the limit)
+static __device__ __align__(256) unsigned char scratch[kNoAllocBytes + (kQueueBytes - kQueueCoreBytes)];
 unsigned char* g_scratch_ptr[kNoAllocDevices] = {};
 std::mutex g_scratch_mu;
 
 size_t noalloc_bytes(const BatchLaunch& bl, int32_t nchunks) {
-    return kQueueBytes + ((order_bufs(nchunks).bytes + 255) & ~size_t(255)) + ((bl.ztab_bytes + 255) & ~size_t(255));
+    return kQueueCoreBytes + ((order_bufs(nchunks).bytes + 255) & ~size_t(255)) + ((bl.ztab_bytes + 255) & ~size_t(255));
 }
 }  // namespace
 

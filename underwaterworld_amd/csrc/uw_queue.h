@@ -17,6 +17,7 @@ constexpr int kResvIndsOffset = 16;  // u64 words from the vertex counter to the
 constexpr int kExitOffset = 32;      // u64 words from the vertex counter to the exit counter
 constexpr size_t kBulkCountByte = 448;
 constexpr size_t kTileCountByte = 512;  // kTileClasses (4) counters
+constexpr size_t kQueueCoreBytes = kTileCountByte;  // the state of launches without the bulk path
 
 // One queued chunk, in queue order (32 bytes, two 16-byte loads): chunk index c (-1: queue
 // empty), resolution n and chunk coordinates. Written by k_place, read once per task.
